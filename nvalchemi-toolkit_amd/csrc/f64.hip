@@ -7,8 +7,8 @@
 // nvalchemi/models/_ops/lj.py:116-216); every configuration it quotes figures on is float32, which
 // is what the tuned kernels of this library serve.  These are the same formulas, in the same order
 // of operations, on doubles: one lane per atom (or LPR lanes per row of the neighbor matrix),
-// coalesced streams, no staging in LDS.  They are bound by HBM like their float32 counterparts and
-// move twice the bytes.
+// coalesced streams, no staging of positions in LDS.  They are bound by HBM like their float32
+// counterparts and move twice the bytes.
 #include "common.h"
 #include "geom.h"
 
@@ -257,7 +257,7 @@ struct Lj64Args {
     const int32_t* shifts;
     const int32_t* nn;
     const int32_t* bidx;
-    int32_t n_atoms, K, fill, half;
+    int32_t n_atoms, K, fill;
     double c4eps, c24eps, sig2, rc2, r_on, inv_sw;
     double* e_atom;   // (N)
     double* forces;   // (N,3)
@@ -273,10 +273,151 @@ __device__ __forceinline__ double group8_sum(double v) {
     return v;
 }
 
-// Full list: a row's owner receives the whole pair force and half the pair energy.  Half list: the
-// kernel runs over the rows as they are and adds the partner's share with atomics (outputs cleared first).
-template <bool HALF>
-__global__ __launch_bounds__(kBlock) void lj_f64_kernel(Lj64Args a) {
+// energy and u'(r)/r of a pair
+__device__ __forceinline__ void lj_f64_pair(const Lj64Args& a, double r2, double& uu, double& gg) {
+    const double ir2 = 1.0 / r2;
+    const double q2 = a.sig2 * ir2, q6 = q2 * q2 * q2, q12 = q6 * q6;
+    uu = a.c4eps * (q12 - q6);
+    gg = -(a.c24eps * (2.0 * q12 - q6)) * ir2;
+    if (a.inv_sw > 0.0) {
+        const double r = sqrt(r2);
+        if (r > a.r_on) {
+            const double t = (r - a.r_on) * a.inv_sw, omt = 1.0 - t;
+            const double S = 1.0 - t * t * t * (10.0 - 15.0 * t + 6.0 * t * t);
+            const double dS = -30.0 * t * t * omt * omt * a.inv_sw;
+            gg = gg * S + uu * dS / r;
+            uu = uu * S;
+        }
+    }
+}
+
+// where the k-th of xx xy xz yy yz zz stands among a system's ten words (energy, then the virial row by row)
+__device__ __forceinline__ int virial_slot(int k) { return k < 3 ? k + 1 : (k < 5 ? k + 2 : 9); }
+
+// Full list: a row's owner receives the whole pair force and half the pair energy.  A workgroup owns a run of rows, eight
+// lanes a row, four entries of a lane in flight (every index and shift, then every position, then the arithmetic: one
+// entry at a time is a chain of two round trips to memory per entry).  Per-system sums are collected in LDS and go to
+// memory once per workgroup and system; one atomic per row on a system's few addresses, as it was, is what the kernel
+// then waits for: 16 clusters of 4000 atoms 645 -> 21 us.
+constexpr int kSysSlots64 = 8;  // consecutive systems a workgroup collects in LDS
+constexpr int kUnroll64 = 4;
+
+template <bool VIRIAL, bool SYS>
+__global__ __launch_bounds__(kBlock) void lj_f64_rows_kernel(Lj64Args a, int rows_per_block) {
+    constexpr int NV = VIRIAL ? 7 : 1;
+    constexpr int G = kBlock / kLpr;
+    __shared__ double s_acc[kSysSlots64][NV];
+    const int row0 = (int)blockIdx.x * rows_per_block;
+    const int row_end = (row0 + rows_per_block) < a.n_atoms ? (row0 + rows_per_block) : a.n_atoms;
+    const int sys_lo = a.bidx[row0];
+    if (SYS) {
+        if (threadIdx.x < kSysSlots64 * NV) (&s_acc[0][0])[threadIdx.x] = 0.0;
+        __syncthreads();
+    }
+    const int sub = threadIdx.x % kLpr;
+    for (int i = row0 + (int)threadIdx.x / kLpr; i < row_end; i += G) {
+        const int sys = a.bidx[i];
+        int cnt = a.nn[i];
+        cnt = cnt < a.K ? cnt : a.K;
+        const double xi = a.pos[3 * (size_t)i], yi = a.pos[3 * (size_t)i + 1], zi = a.pos[3 * (size_t)i + 2];
+        const int32_t* row = a.nm + (size_t)i * a.K;
+        const int32_t* srow = a.shifts ? a.shifts + (size_t)i * a.K * 3 : nullptr;
+        double h[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) h[k] = (a.shifts && a.cells) ? a.cells[9 * (size_t)sys + k] : 0.0;
+        double e = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+        double w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // xx xy xz yy yz zz
+        for (int k0 = 0; k0 < cnt; k0 += kLpr * kUnroll64) {
+            int jj[kUnroll64], s0[kUnroll64], s1[kUnroll64], s2[kUnroll64];
+            double xj[kUnroll64], yj[kUnroll64], zj[kUnroll64];
+#pragma unroll
+            for (int u = 0; u < kUnroll64; ++u) {
+                // (clamped, unconditional loads: slot cnt - 1 exists)
+                const int k = k0 + u * kLpr + sub, kq = k < cnt ? k : cnt - 1;
+                jj[u] = row[kq];
+                s0[u] = s1[u] = s2[u] = 0;
+                if (srow) {
+                    s0[u] = srow[3 * kq + 0];
+                    s1[u] = srow[3 * kq + 1];
+                    s2[u] = srow[3 * kq + 2];
+                }
+                if (k >= cnt) jj[u] = -1;
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll64; ++u) {
+                const bool ok = jj[u] >= 0 && jj[u] < a.fill;
+                const double* pj = a.pos + 3 * (size_t)(ok ? jj[u] : i);
+                if (!ok) jj[u] = -1;
+                xj[u] = pj[0];
+                yj[u] = pj[1];
+                zj[u] = pj[2];
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll64; ++u) {
+                double d0, d1, d2;
+                const double r2 = pair_d2_exact(xi, yi, zi, xj[u], yj[u], zj[u], s0[u], s1[u], s2[u], h, d0, d1, d2);
+                if (jj[u] < 0 || !(r2 < a.rc2)) continue;
+                double uu, gg;
+                lj_f64_pair(a, r2, uu, gg);
+                e += 0.5 * uu;
+                fx += gg * d0;
+                fy += gg * d1;
+                fz += gg * d2;
+                if (VIRIAL) {
+                    const double hg = -0.5 * gg;
+                    w[0] += hg * d0 * d0;
+                    w[1] += hg * d0 * d1;
+                    w[2] += hg * d0 * d2;
+                    w[3] += hg * d1 * d1;
+                    w[4] += hg * d1 * d2;
+                    w[5] += hg * d2 * d2;
+                }
+            }
+        }
+        e = group8_sum(e);
+        fx = group8_sum(fx);
+        fy = group8_sum(fy);
+        fz = group8_sum(fz);
+        if (VIRIAL) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) w[k] = group8_sum(w[k]);
+        }
+        if (sub != 0) continue;
+        a.e_atom[i] = e;
+        a.forces[3 * (size_t)i + 0] = fx;
+        a.forces[3 * (size_t)i + 1] = fy;
+        a.forces[3 * (size_t)i + 2] = fz;
+        if (SYS) {
+            const unsigned slot = (unsigned)(sys - sys_lo);
+            if (slot < (unsigned)kSysSlots64) {
+                atomicAdd(&s_acc[slot][0], e);
+                if (VIRIAL) {
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) atomicAdd(&s_acc[slot][1 + k], w[k]);
+                }
+            } else {
+                double* out = a.sys_acc + 10 * (size_t)sys;
+                atomic_add_f64(out, e);
+                if (VIRIAL) {
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) atomic_add_f64(out + virial_slot(k), w[k]);
+                }
+            }
+        }
+    }
+    if (SYS) {
+        __syncthreads();
+        if (threadIdx.x < kSysSlots64 * NV) {
+            const int slot = threadIdx.x / NV, k = threadIdx.x % NV;
+            const double v = s_acc[slot][k];
+            // (a slot that no row touched is still zero and names a system that may not exist)
+            if (v != 0.0) atomic_add_f64(a.sys_acc + 10 * (size_t)(sys_lo + slot) + (k == 0 ? 0 : virial_slot(k - 1)), v);
+        }
+    }
+}
+
+// Half list: the kernel runs over the rows as they are and adds the partner's share with atomics (outputs cleared first).
+__global__ __launch_bounds__(kBlock) void lj_f64_half_kernel(Lj64Args a) {
     const int i = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kLpr);
     const int sub = threadIdx.x % kLpr;
     if (i >= a.n_atoms) return;  // (whole groups of 8 lanes leave together)
@@ -303,31 +444,17 @@ __global__ __launch_bounds__(kBlock) void lj_f64_kernel(Lj64Args a) {
         const double r2 = pair_d2_exact(xi, yi, zi, a.pos[3 * (size_t)j], a.pos[3 * (size_t)j + 1],
                                         a.pos[3 * (size_t)j + 2], s0, s1, s2, h, d0, d1, d2);
         if (!(r2 < a.rc2)) continue;
-        const double ir2 = 1.0 / r2;
-        const double q2 = a.sig2 * ir2, q6 = q2 * q2 * q2, q12 = q6 * q6;
-        double uu = a.c4eps * (q12 - q6);
-        double gg = -(a.c24eps * (2.0 * q12 - q6)) * ir2;  // u'(r)/r
-        if (a.inv_sw > 0.0) {
-            const double r = sqrt(r2);
-            if (r > a.r_on) {
-                const double t = (r - a.r_on) * a.inv_sw, omt = 1.0 - t;
-                const double S = 1.0 - t * t * t * (10.0 - 15.0 * t + 6.0 * t * t);
-                const double dS = -30.0 * t * t * omt * omt * a.inv_sw;
-                gg = gg * S + uu * dS / r;
-                uu = uu * S;
-            }
-        }
+        double uu, gg;
+        lj_f64_pair(a, r2, uu, gg);
         e += 0.5 * uu;
         fx += gg * d0;
         fy += gg * d1;
         fz += gg * d2;
-        if (HALF) {
-            atomic_add_f64(a.e_atom + j, 0.5 * uu);
-            atomic_add_f64(a.forces + 3 * (size_t)j + 0, -gg * d0);
-            atomic_add_f64(a.forces + 3 * (size_t)j + 1, -gg * d1);
-            atomic_add_f64(a.forces + 3 * (size_t)j + 2, -gg * d2);
-        }
-        const double hg = HALF ? -gg : -0.5 * gg;
+        atomic_add_f64(a.e_atom + j, 0.5 * uu);
+        atomic_add_f64(a.forces + 3 * (size_t)j + 0, -gg * d0);
+        atomic_add_f64(a.forces + 3 * (size_t)j + 1, -gg * d1);
+        atomic_add_f64(a.forces + 3 * (size_t)j + 2, -gg * d2);
+        const double hg = -gg;
         w[0] += hg * d0 * d0;
         w[1] += hg * d0 * d1;
         w[2] += hg * d0 * d2;
@@ -344,20 +471,13 @@ __global__ __launch_bounds__(kBlock) void lj_f64_kernel(Lj64Args a) {
         for (int k = 0; k < 6; ++k) w[k] = group8_sum(w[k]);
     }
     if (sub != 0) return;
-    if (HALF) {
-        atomic_add_f64(a.e_atom + i, e);
-        atomic_add_f64(a.forces + 3 * (size_t)i + 0, fx);
-        atomic_add_f64(a.forces + 3 * (size_t)i + 1, fy);
-        atomic_add_f64(a.forces + 3 * (size_t)i + 2, fz);
-    } else {
-        a.e_atom[i] = e;
-        a.forces[3 * (size_t)i + 0] = fx;
-        a.forces[3 * (size_t)i + 1] = fy;
-        a.forces[3 * (size_t)i + 2] = fz;
-    }
+    atomic_add_f64(a.e_atom + i, e);
+    atomic_add_f64(a.forces + 3 * (size_t)i + 0, fx);
+    atomic_add_f64(a.forces + 3 * (size_t)i + 1, fy);
+    atomic_add_f64(a.forces + 3 * (size_t)i + 2, fz);
     if (a.sys_acc) {
         double* out = a.sys_acc + 10 * (size_t)sys;
-        // (full list: a system's energy is the sum of its atoms' energies, added below once they are final)
+        // (a system's energy is the sum of its atoms' energies, added below once they are final)
         atomic_add_f64(out + 1, w[0]);
         atomic_add_f64(out + 2, w[1]);
         atomic_add_f64(out + 3, w[2]);
@@ -657,7 +777,6 @@ NVAMD_EXPORT int32_t nvamd_lj_energy_forces_f64(const double* positions, const d
     a.n_atoms = n_atoms;
     a.K = max_neighbors;
     a.fill = fill_value < n_atoms ? fill_value : n_atoms;
-    a.half = half_list ? 1 : 0;
     a.c4eps = 4.0 * epsilon;
     a.c24eps = 24.0 * epsilon;
     a.sig2 = sigma * sigma;
@@ -676,13 +795,20 @@ NVAMD_EXPORT int32_t nvamd_lj_energy_forces_f64(const double* positions, const d
         if (half_list) {
             hipLaunchKernelGGL(lj_f64_clear_kernel, blocks((size_t)n_atoms), blk, 0, st, atomic_energies, (size_t)n_atoms);
             hipLaunchKernelGGL(lj_f64_clear_kernel, blocks((size_t)n_atoms * 3), blk, 0, st, forces, (size_t)n_atoms * 3);
-            hipLaunchKernelGGL(lj_f64_kernel<true>, blocks((size_t)n_atoms * kLpr), blk, 0, st, a);
+            hipLaunchKernelGGL(lj_f64_half_kernel, blocks((size_t)n_atoms * kLpr), blk, 0, st, a);
+            if (a.sys_acc)
+                hipLaunchKernelGGL(lj_f64_sys_energy_kernel, blocks((size_t)n_atoms), blk, 0, st, atomic_energies,
+                                   batch_idx, a.sys_acc, n_atoms);
         } else {
-            hipLaunchKernelGGL(lj_f64_kernel<false>, blocks((size_t)n_atoms * kLpr), blk, 0, st, a);
+            // runs of 32 rows (one pass of a workgroup) up to 64 k rows, longer ones from there on: enough workgroups to
+            // fill the chip several times over, few enough atomics per system
+            int rows = kBlock / kLpr;
+            while (rows < 512 && (n_atoms + rows - 1) / rows > 2048) rows *= 2;
+            const dim3 grid((unsigned)((n_atoms + rows - 1) / rows));
+            if (virials) hipLaunchKernelGGL((lj_f64_rows_kernel<true, true>), grid, blk, 0, st, a, rows);
+            else if (a.sys_acc) hipLaunchKernelGGL((lj_f64_rows_kernel<false, true>), grid, blk, 0, st, a, rows);
+            else hipLaunchKernelGGL((lj_f64_rows_kernel<false, false>), grid, blk, 0, st, a, rows);
         }
-        if (a.sys_acc)
-            hipLaunchKernelGGL(lj_f64_sys_energy_kernel, blocks((size_t)n_atoms), blk, 0, st, atomic_energies, batch_idx,
-                               a.sys_acc, n_atoms);
     }
     if (want_sys && n_systems > 0)
         hipLaunchKernelGGL(lj_f64_finish_kernel, blocks((size_t)n_systems * 10), blk, 0, st, a.sys_acc, system_energies,

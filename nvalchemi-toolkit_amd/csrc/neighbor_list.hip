@@ -735,13 +735,25 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_part, int* tot
     return before + incl - v;
 }
 
+template <bool F64>
+struct PosType {
+    using type = float;
+    static __device__ __forceinline__ const float* of(const NlArgs& a) { return a.pos; }
+};
+template <>
+struct PosType<true> {
+    using type = double;
+    static __device__ __forceinline__ const double* of(const NlArgs& a) { return a.pos64; }
+};
+
 // kKeep: atoms per thread whose positions and bins stay in registers from the histogram to the scatter (systems of
 // up to kKeep * kSortBlock atoms are binned once): four, or eight when the mean system has more than 2048 atoms.
 // kWaves: waves per SIMD the kernel is built for.  With more systems than CUs the instance of four atoms is held to
 // 128 registers (four waves per SIMD, two workgroups per CU: one system's chain of dependent steps then runs
 // beside another's, 6 % off the build of 2048 mixed systems for 19 spilled words); with fewer systems than that
 // nothing would run beside it, and it keeps its 152 registers (the spills cost 64 boxes of 500 atoms 2 %).
-template <int kKeep, int kWaves>
+// F64: the type of the positions.
+template <int kKeep, int kWaves, bool F64>
 __global__ __launch_bounds__(kSortBlock, kWaves) void nl_system_sort_kernel(NlArgs a, NlWorkspace ws) {
     __shared__ NlSys s_sys;
     __shared__ uint32_t s_bounds[6];
@@ -756,15 +768,17 @@ __global__ __launch_bounds__(kSortBlock, kWaves) void nl_system_sort_kernel(NlAr
     const int slot = __builtin_amdgcn_readfirstlane(ws.hdr->flip);
     if (t == 0 && tid == 0) retire_other_slot(ws.hdr);
     const int begin = a.ptr[t], end = a.ptr[t + 1];
+    // nothing to search: no cells, no units, and nobody looks at the system's records
+    if (end <= begin || (a.rebuild && !a.rebuild[t])) return;
     // up to kKeep atoms per thread stay in registers from here to the scatter; their positions
-    // are requested now, so that they arrive while thread 0 works out the system's grid
-    const bool kept = !a.pos64 && (end - begin) <= kKeep * kSortBlock;
-    float my_pos[kKeep][3];
+    // are requested now, so that they arrive while the first wave works out the system's axes
+    const bool kept = (end - begin) <= kKeep * kSortBlock;
+    typename PosType<F64>::type my_pos[kKeep][3];
     if (kept) {
 #pragma unroll
         for (int k = 0; k < kKeep; ++k) {
             const int i = begin + tid + k * kSortBlock;
-            const float* r = a.pos + 3 * (size_t)(i < end ? i : (end > begin ? begin : 0));
+            const auto* r = PosType<F64>::of(a) + 3 * (size_t)(i < end ? i : begin);
             my_pos[k][0] = r[0];
             my_pos[k][1] = r[1];
             my_pos[k][2] = r[2];
@@ -779,25 +793,49 @@ __global__ __launch_bounds__(kSortBlock, kWaves) void nl_system_sort_kernel(NlAr
     }
     __syncthreads();
     const int cell_base = begin + (kMinCellCap + 1) * t;
-    const bool idle = end <= begin || (a.rebuild && !a.rebuild[t]);  // nothing to search: no cells, no units
     // ---- bounds on non-periodic axes
-    if (!idle && !(s_sys.per[0] && s_sys.per[1] && s_sys.per[2])) {
-        for (int i = begin + tid; i < end; i += kSortBlock) {
+    // (each thread over its own atoms, then over its wave, then one LDS atomic per wave and bound: with an LDS atomic per
+    // atom on the same six words, and float64 positions binned twice, the sort of 16 open clusters of 4000 atoms took
+    // 114 us instead of 20, that of eight open molecules 13.6 instead of 10.7)
+    if (!(s_sys.per[0] && s_sys.per[1] && s_sys.per[2])) {
+        uint32_t lo[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, hi[3] = {0u, 0u, 0u};
+        auto widen = [&](const Pos3& r) {
             double f[3];
-            frac_of(s_sys, load_pos(a, (size_t)i), f);
+            frac_of(s_sys, r, f);
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                if (s_sys.per[d]) continue;
-                float lo = __double2float_rd(f[d]), hi = __double2float_ru(f[d]);
-                atomicMin(&s_bounds[d], float_order_key(lo));
-                atomicMax(&s_bounds[3 + d], float_order_key(hi));
+                const uint32_t below = float_order_key(__double2float_rd(f[d])), above = float_order_key(__double2float_ru(f[d]));
+                lo[d] = below < lo[d] ? below : lo[d];
+                hi[d] = above > hi[d] ? above : hi[d];
+            }
+        };
+        if (kept) {
+#pragma unroll
+            for (int k = 0; k < kKeep; ++k)
+                if (begin + tid + k * kSortBlock < end)
+                    widen(Pos3{(double)my_pos[k][0], (double)my_pos[k][1], (double)my_pos[k][2]});
+        } else {
+            for (int i = begin + tid; i < end; i += kSortBlock) widen(load_pos(a, (size_t)i));
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (s_sys.per[d]) continue;
+#pragma unroll
+            for (int o = kWave / 2; o > 0; o >>= 1) {
+                const uint32_t l = (uint32_t)__shfl_xor((int)lo[d], o, kWave), h = (uint32_t)__shfl_xor((int)hi[d], o, kWave);
+                lo[d] = l < lo[d] ? l : lo[d];
+                hi[d] = h > hi[d] ? h : hi[d];
+            }
+            if (lane_id() == 0 && lo[d] <= hi[d]) {
+                atomicMin(&s_bounds[d], lo[d]);
+                atomicMax(&s_bounds[3 + d], hi[d]);
             }
         }
         __syncthreads();
     }
     // ---- grid
     if (first_wave) {
-        system_grid(s_sys, s_view, axes, a, idle ? 0 : end - begin, s_bounds, &s_err, cell_base);
+        system_grid(s_sys, s_view, axes, a, end - begin, s_bounds, &s_err, cell_base);
         if (tid == 0) {
             ws.cell_offset[t] = cell_base;
             if (s_err) atomicOr(&ws.hdr->error[slot], s_err);
@@ -813,7 +851,6 @@ __global__ __launch_bounds__(kSortBlock, kWaves) void nl_system_sort_kernel(NlAr
         int* view_out = reinterpret_cast<int*>(ws.ssys + t);
         for (int w = tid; w < (int)(sizeof(NlSearchSys) / sizeof(int)); w += kSortBlock) view_out[w] = view[w];
     }
-    if (idle) return;
     const int n_cells = s_sys.n_cells;
     const bool in_lds = n_cells <= kSortCells;
     int* g_hist = ws.cell_count + cell_base;
@@ -1753,12 +1790,17 @@ static int32_t nl_build_impl(const float* positions, const float* cell, const do
                                                             : (sort_path == NVAMD_NL_SORT_PER_SYSTEM);
     if (per_system) {
         // many small systems: set-up to scatter in one workgroup per system
-        if (!a.pos64 && n_atoms / n_systems > 4 * kSortBlock && n_atoms / n_systems <= 8 * kSortBlock)
-            hipLaunchKernelGGL((nl_system_sort_kernel<8, 2>), dim3(n_systems), dim3(kSortBlock), 0, st, a, ws);
-        else if (n_systems > 256)
-            hipLaunchKernelGGL((nl_system_sort_kernel<4, 4>), dim3(n_systems), dim3(kSortBlock), 0, st, a, ws);
-        else
-            hipLaunchKernelGGL((nl_system_sort_kernel<4, 2>), dim3(n_systems), dim3(kSortBlock), 0, st, a, ws);
+#define NVAMD_NL_SORT(K, W)                                                                                        \
+    if (a.pos64) hipLaunchKernelGGL((nl_system_sort_kernel<K, W, true>), dim3(n_systems), dim3(kSortBlock), 0, st, a, ws); \
+    else hipLaunchKernelGGL((nl_system_sort_kernel<K, W, false>), dim3(n_systems), dim3(kSortBlock), 0, st, a, ws)
+        if (n_atoms / n_systems > 4 * kSortBlock && n_atoms / n_systems <= 8 * kSortBlock) {
+            NVAMD_NL_SORT(8, 2);
+        } else if (n_systems > 256) {
+            NVAMD_NL_SORT(4, 4);
+        } else {
+            NVAMD_NL_SORT(4, 2);
+        }
+#undef NVAMD_NL_SORT
     } else {
         const size_t n_prep = (size_t)ws.max_cells;
         const size_t n_waves = (size_t)n_systems * kWave;
