@@ -38,6 +38,17 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
+// rows of two or three 32-bit words: one 8- or 12-byte access each (4-byte alignment is all it needs)
+struct Int2 {
+    int x, y;
+};
+struct Int3 {
+    int x, y, z;
+};
+struct Float3 {
+    float x, y, z;
+};
+
 // wave-wide sum of a double via xor shuffles (all 64 lanes end with the total)
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

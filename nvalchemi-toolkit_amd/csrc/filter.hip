@@ -11,9 +11,8 @@
 // reference evaluates it in float32, so the two can differ only for pairs within float32
 // rounding of the cutoff.
 //
-// Bound: HBM, 16 B read and up to 16 B written per slot plus one gathered position per valid
-// slot.  One wavefront per row: 64 slots per step, a ballot and a prefix count give every kept
-// entry its place.
+// Bound: HBM, 4 B read per slot, 12 B more and one gathered position per valid slot, 16 B written per slot.  One wavefront
+// per row: 256 slots in flight, a ballot and a prefix count give every kept entry its place.
 #include "common.h"
 #include "geom.h"
 
@@ -21,7 +20,25 @@ namespace nvamd {
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kInFlight = 4;  // steps of 64 slots whose loads are in flight together
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// Words [begin, end) of a row of int32 set to one value by a wave, in 16-byte stores between the aligned addresses.
+// (non-temporal: nobody reads the padding back, and it is most of what is written)
+__device__ __forceinline__ void fill_words(int32_t* row, int begin, int end, int value, int lane) {
+    const int to_line = (int)((0 - (reinterpret_cast<uintptr_t>(row + begin) >> 2)) & 3);
+    const int first = begin + to_line < end ? begin + to_line : end;
+    const int last = first + ((end - first) & ~3);
+    if (begin + lane < first) __builtin_nontemporal_store(value, row + begin + lane);
+    const v4i v = {value, value, value, value};
+    for (int k = first + 4 * lane; k < last; k += 4 * kWave) __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(row + k));
+    if (last + lane < end) __builtin_nontemporal_store(value, row + last + lane);
+}
+
+// The shift of a padding slot is not read (it is zero in the result whatever it was), the four steps' loads go out
+// together, and the padding leaves in 16-byte stores: 64 000 rows of 272 slots (78 valid) take 87 us instead of 124, 60 when
+// they have just been read (408 MB have to move: 4.7 TB/s).
 __global__ __launch_bounds__(kBlock) void filter_matrix_kernel(const float* __restrict__ pos,
                                                                const float* __restrict__ cells, int cell_stride,
                                                                const int32_t* __restrict__ nm,
@@ -30,58 +47,58 @@ __global__ __launch_bounds__(kBlock) void filter_matrix_kernel(const float* __re
                                                                int fill, double rc2, int32_t* __restrict__ out_nm,
                                                                int32_t* __restrict__ out_nn,
                                                                int32_t* __restrict__ out_shifts) {
-    const int i = (int)((blockIdx.x * (size_t)kBlock + threadIdx.x) / kWave);
+    const int i = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)kBlock + threadIdx.x) / kWave));
     if (i >= n_atoms) return;
     const int lane = lane_id();
     const float xi = pos[3 * (size_t)i], yi = pos[3 * (size_t)i + 1], zi = pos[3 * (size_t)i + 2];
     const bool shifted = cells != nullptr && shifts != nullptr;
     const float* cell = shifted ? cells + (size_t)cell_stride * (bidx ? bidx[i] : 0) : nullptr;
     const int32_t* row = nm + (size_t)i * K;
-    const int32_t* srow = shifts ? shifts + (size_t)i * K * 3 : nullptr;
+    const Int3* srow = shifts ? reinterpret_cast<const Int3*>(shifts) + (size_t)i * K : nullptr;
     int32_t* orow = out_nm + (size_t)i * K;
     int32_t* osrow = out_shifts ? out_shifts + (size_t)i * K * 3 : nullptr;
     int kept = 0;
-    for (int k0 = 0; k0 < K; k0 += kWave) {
-        const int k = k0 + lane;
-        bool keep = false;
-        int j = fill, s0 = 0, s1 = 0, s2 = 0;
-        if (k < K) {
-            j = row[k];
-            if (srow) {
-                s0 = srow[3 * k + 0];
-                s1 = srow[3 * k + 1];
-                s2 = srow[3 * k + 2];
-            }
-            if (j < fill) {
+    for (int k0 = 0; k0 < K; k0 += kInFlight * kWave) {
+        int j[kInFlight];
+        Int3 s[kInFlight];
+        Float3 p[kInFlight];
+#pragma unroll
+        for (int q = 0; q < kInFlight; ++q) {
+            const int k = k0 + q * kWave + lane;
+            j[q] = fill;
+            if (k < K) j[q] = row[k];
+        }
+#pragma unroll
+        for (int q = 0; q < kInFlight; ++q) {
+            s[q] = Int3{0, 0, 0};
+            p[q] = Float3{0.f, 0.f, 0.f};
+            if (j[q] < fill) {
+                if (srow) s[q] = srow[k0 + q * kWave + lane];
                 // (the reference clamps the index into range before the gather)
-                const int js = j < 0 ? 0 : (j >= n_atoms ? n_atoms - 1 : j);
-                const float* pj = pos + 3 * (size_t)js;
+                const int js = j[q] < 0 ? 0 : (j[q] >= n_atoms ? n_atoms - 1 : j[q]);
+                p[q] = reinterpret_cast<const Float3*>(pos)[js];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kInFlight; ++q) {
+            bool keep = false;
+            if (j[q] < fill) {
                 double tx = 0.0, ty = 0.0, tz = 0.0, d0, d1, d2;
-                if (shifted) shift_vector(cell, s0, s1, s2, tx, ty, tz);
-                keep = pair_d2_shifted(xi, yi, zi, pj[0], pj[1], pj[2], tx, ty, tz, d0, d1, d2) < rc2;
+                if (shifted) shift_vector(cell, s[q].x, s[q].y, s[q].z, tx, ty, tz);
+                keep = pair_d2_shifted(xi, yi, zi, p[q].x, p[q].y, p[q].z, tx, ty, tz, d0, d1, d2) < rc2;
             }
-        }
-        const unsigned long long m = __ballot(keep);
-        if (keep) {
-            const int at = kept + __popcll(m & ((1ull << lane) - 1ull));
-            orow[at] = j;
-            if (osrow) {
-                osrow[3 * at + 0] = s0;
-                osrow[3 * at + 1] = s1;
-                osrow[3 * at + 2] = s2;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+            if (keep) {
+                const int at = kept + __popcll(m & ((1ull << lane) - 1ull));
+                orow[at] = j[q];
+                if (osrow) reinterpret_cast<Int3*>(osrow)[at] = s[q];
             }
+            kept += __popcll(m);
         }
-        kept += __popcll(m);
     }
     // the rest of the row is padding
-    for (int k = kept + lane; k < K; k += kWave) {
-        orow[k] = fill;
-        if (osrow) {
-            osrow[3 * k + 0] = 0;
-            osrow[3 * k + 1] = 0;
-            osrow[3 * k + 2] = 0;
-        }
-    }
+    fill_words(orow, kept, K, fill, lane);
+    if (osrow) fill_words(osrow, 3 * kept, 3 * K, 0, lane);
     if (lane == 0) out_nn[i] = kept;
 }
 
