@@ -582,6 +582,41 @@ int32_t nvamd_put_masked_segmented(const void* source, const int32_t* source_bat
                                    int32_t num_systems, int32_t total_rows, int64_t row_bytes,
                                    void* workspace, size_t workspace_bytes, void* stream);
 
+/* Batch.put (nvalchemi/data/batch.py:876-985) as one plan and one copy: the masked systems that fit on every level (a free
+ * slot among the rows with one per system, room behind the last segment of each segmented level) move, all tensors
+ * together.  What the calls above do level by level and tensor by tensor, with the same result. */
+typedef struct {
+    const void* source;  /* first row */
+    void* dest;
+    int64_t row_bytes;
+    int32_t level;        /* 0: a row per system; 1, 2: rows of segmented level 0, 1 */
+    int32_t source_rows;  /* rows of `source` (no more than that are read) */
+} nvamd_put_field;
+
+typedef struct {
+    const int32_t* source_ptr; /* (num_systems + 1) */
+    const int32_t* dest_ptr;   /* (num_dest + 1) boundaries of the segments that are there */
+    int32_t* new_ptr;          /* (new_ptr_entries >= num_dest + num_systems + 1) out: all boundaries, zeros behind them */
+    int32_t* new_lengths;      /* (num_dest + num_systems) out: lengths of the segments */
+    int32_t num_dest;
+    int32_t capacity;          /* rows of the destination */
+    int32_t new_ptr_entries;
+    int32_t max_length;        /* a masked segment longer than this refuses the whole call (-1: no such limit) */
+} nvamd_put_level;
+
+/* copied[i] = 1 / 0 for the systems that moved / did not (may be source_mask itself); dest_mask (n_slots; null: all free, and
+ * none is marked) gets the filled slots; counts (8): masked systems, longest masked segment of level 0, of level 1,
+ * systems moved, 1 unless refused.  A refused call (more masked systems than max_masked >= 0, or a segment longer than its
+ * level allows) writes only counts.  n_slots < 0: there are no rows with one per system. */
+int32_t nvamd_put_batch(const nvamd_put_field* fields, int32_t n_fields, const nvamd_put_level* levels, int32_t n_levels,
+                        const uint8_t* source_mask, uint8_t* copied, uint8_t* dest_mask, int32_t num_systems,
+                        int32_t n_slots, int32_t max_masked, int32_t* counts, void* workspace, size_t workspace_bytes,
+                        void* stream);
+
+/* `n` byte ranges copied / set to zero in one launch for up to 48 of them (ranges must not overlap). */
+int32_t nvamd_copy_ranges(const void* const* source, void* const* dest, const int64_t* bytes, int32_t n, void* stream);
+int32_t nvamd_zero_ranges(void* const* dest, const int64_t* bytes, int32_t n, void* stream);
+
 /* compute_put_fit_mask_segmented (buffer_kernels.py:500-610): fit_mask[i] = segment i would be
  * copied by the call above.  (The reference's host wrapper clears the mask instead when
  * dest_batch_ptr is too short; that check stays with the caller.) */

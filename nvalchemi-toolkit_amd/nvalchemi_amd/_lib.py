@@ -24,6 +24,16 @@ _vp = _c.c_void_p
 _i32 = _c.c_int32
 _f64 = _c.c_double
 
+
+class PutField(_c.Structure):
+    _fields_ = [("source", _vp), ("dest", _vp), ("row_bytes", _c.c_int64), ("level", _i32), ("source_rows", _i32)]
+
+
+class PutLevel(_c.Structure):
+    _fields_ = [("source_ptr", _vp), ("dest_ptr", _vp), ("new_ptr", _vp), ("new_lengths", _vp), ("num_dest", _i32),
+                ("capacity", _i32), ("new_ptr_entries", _i32), ("max_length", _i32)]
+
+
 _SIGNATURES = {
     "nvamd_abi_version": (_i32, []),
     "nvamd_last_error": (_c.c_char_p, []),
@@ -89,6 +99,10 @@ _SIGNATURES = {
     "nvamd_defrag_per_system": (_i32, [_vp, _vp, _i32, _c.c_int64, _vp, _c.c_size_t, _vp]),
     "nvamd_put_masked_segmented": (_i32, [_vp] * 5 + [_i32, _i32, _vp, _vp, _i32, _i32, _c.c_int64, _vp,
                                           _c.c_size_t, _vp]),
+    "nvamd_put_batch": (_i32, [_c.POINTER(PutField), _i32, _c.POINTER(PutLevel), _i32, _vp, _vp, _vp, _i32, _i32, _i32, _vp,
+                               _vp, _c.c_size_t, _vp]),
+    "nvamd_copy_ranges": (_i32, [_c.POINTER(_vp), _c.POINTER(_vp), _c.POINTER(_c.c_int64), _i32, _vp]),
+    "nvamd_zero_ranges": (_i32, [_c.POINTER(_vp), _c.POINTER(_c.c_int64), _i32, _vp]),
     "nvamd_put_fit_mask_segmented": (_i32, [_vp] * 3 + [_i32, _i32, _vp, _i32, _vp, _c.c_size_t, _vp]),
     "nvamd_defrag_segmented": (_i32, [_vp] * 4 + [_i32, _i32, _c.c_int64, _vp, _c.c_size_t, _vp]),
 }
@@ -768,6 +782,51 @@ def defrag_segmented(source, source_batch_ptr, source_data_copied, num_kept) -> 
         sp, _dev(source_batch_ptr, "source_batch_ptr", torch.int32, (n + 1,)),
         _mask(source_data_copied, "source_data_copied", n), _dev(num_kept, "num_kept", torch.int32, (1,)),
         n, rows, rb, ws.data_ptr(), ws.numel(), _stream(source.device)), "nvamd_defrag_segmented")
+
+
+def plain_on_device(t: torch.Tensor, device: torch.device) -> bool:
+    """A tensor whose rows may be moved through its pointer: an ordinary contiguous one of a supported dtype on ``device``
+    that no gradient is recorded for."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.device == device and t.dtype in BUFFER_DTYPES
+            and not t.requires_grad and t.is_contiguous())
+
+
+def put_batch(fields, levels, mask, copied, dest_mask, n_slots: int, max_masked: int, counts) -> None:
+    """``fields``: (source, dest, row bytes, level, source rows) each; ``levels``: (source ptr, dest ptr, new ptr, new lengths,
+    segments there, capacity, longest segment allowed) each.  The caller has looked at shapes, dtypes and devices."""
+    dev, n = mask.device, mask.shape[0]
+    f = (PutField * max(len(fields), 1))(*[PutField(s.data_ptr(), d.data_ptr(), rb, lv, rows) for s, d, rb, lv, rows in fields])
+    q = (PutLevel * max(len(levels), 1))(*[
+        PutLevel(_dev(sp, "source_ptr", torch.int32, (n + 1,)), _dev(dp, "dest_ptr", torch.int32), new.data_ptr(),
+                 lengths.data_ptr(), nd, cap, new.shape[0], longest) for sp, dp, new, lengths, nd, cap, longest in levels])
+    ws = workspaces.get(dev, "buffers", 13 * n + 512)
+    _check(library().nvamd_put_batch(
+        f, len(fields), q, len(levels), _mask(mask, "mask", n), _mask(copied, "copied", n),
+        None if dest_mask is None else _mask(dest_mask, "dest_mask", n_slots), n, n_slots, max_masked,
+        _dev(counts, "counts", torch.int32, (8,)), ws.data_ptr(), ws.numel(), _stream(dev)), "nvamd_put_batch")
+    torch.autograd.graph.increment_version([d for _, d, _, _, _ in fields] + [copied] + ([] if dest_mask is None else [dest_mask]))
+
+
+def _ranges(tensors):
+    n = len(tensors)
+    return (_vp * n)(*[t.data_ptr() for t in tensors])
+
+
+def copy_tensors(sources, dests) -> None:
+    """``dest.copy_(source)`` for pairs of equal shape and dtype (contiguous, on one device), in one launch."""
+    n = len(sources)
+    if n:
+        sizes = (_c.c_int64 * n)(*[t.numel() * t.element_size() for t in sources])
+        _check(library().nvamd_copy_ranges(_ranges(sources), _ranges(dests), sizes, n, _stream(dests[0].device)), "nvamd_copy_ranges")
+
+
+def zero_tensors(tensors) -> None:
+    """``zero_()`` of contiguous tensors on one device, in one launch."""
+    n = len(tensors)
+    if n:
+        sizes = (_c.c_int64 * n)(*[t.numel() * t.element_size() for t in tensors])
+        _check(library().nvamd_zero_ranges(_ranges(tensors), sizes, n, _stream(tensors[0].device)), "nvamd_zero_ranges")
+        torch.autograd.graph.increment_version(tensors)
 
 
 # --------------------------------------------------------------------------------------------

@@ -12,9 +12,12 @@ writes routed by key name with unknown names going to the system group
 
 from __future__ import annotations
 
+import math
 from typing import Any, Iterator
 
 import torch
+
+from nvalchemi_amd import _lib
 
 from . import buffer_kernels
 from .atomic_data import EDGE_KEYS, NODE_KEYS, SYSTEM_KEYS, AtomicData
@@ -29,6 +32,34 @@ def _bool_on(mask: torch.Tensor, device) -> torch.Tensor:
     reach the caller), else a converted copy."""
     return mask if mask.dtype == torch.bool and mask.device == torch.device(device) else mask.to(
         device=device, dtype=torch.bool)
+
+
+def _span(idx: list[int]) -> tuple[int, int] | None:
+    """``(first, end)`` when ``idx`` counts up one by one."""
+    lo, hi = idx[0], idx[0] + len(idx)
+    return (lo, hi) if idx == list(range(lo, hi)) else None
+
+
+def _copies(tensors: list[torch.Tensor]) -> list[torch.Tensor]:
+    """Contiguous copies (one launch for tensors on the GPU that need no gradient)."""
+    dev = tensors[0].device if tensors else None
+    if dev is None or dev.type != "cuda" or torch.compiler.is_compiling() \
+            or not all(_lib.plain_on_device(t, dev) for t in tensors):
+        return [t.clone(memory_format=torch.contiguous_format) for t in tensors]
+    out = [torch.empty(t.shape, dtype=t.dtype, device=dev) for t in tensors]
+    _lib.copy_tensors(tensors, out)
+    return out
+
+
+def _zero_all(tensors: list[torch.Tensor]) -> None:
+    """``zero_()`` of every tensor (one launch where :func:`_copies` makes one)."""
+    dev = tensors[0].device if tensors else None
+    if dev is None or dev.type != "cuda" or torch.compiler.is_compiling() \
+            or not all(_lib.plain_on_device(t, dev) for t in tensors):
+        for t in tensors:
+            t.zero_()
+    else:
+        _lib.zero_tensors(tensors)
 
 
 class SegmentedGroup:
@@ -144,6 +175,15 @@ class SegmentedGroup:
         lengths_host = self.lengths_list()
         new_lengths = [lengths_host[i] for i in idx]
         total = sum(new_lengths)
+        span = _span(idx)
+        if span is not None:  # (one slice per tensor)
+            start = sum(lengths_host[: span[0]])
+            names = list(self._tensors)
+            parts = _copies([self._tensors[k][start: start + total] for k in names]
+                            + [self.segment_lengths[span[0]: span[1]]])
+            out = SegmentedGroup(dict(zip(names, parts)), parts[-1], self.device)
+            out._lengths_host = new_lengths
+            return out
         sel = torch.tensor(idx, dtype=torch.long, device=self.device)
         lens = self.segment_lengths[sel].to(torch.long)
         starts = self.batch_ptr[sel].to(torch.long)
@@ -267,8 +307,10 @@ class SegmentedGroup:
 
     def zero(self) -> None:
         """No segments, all rows zero; tensors and boundary headroom are kept."""
-        for t in self._tensors.values():
-            t.zero_()
+        _zero_all(list(self._tensors.values()))
+        self._no_segments()
+
+    def _no_segments(self) -> None:
         self.segment_lengths = torch.empty(0, dtype=torch.int32, device=self.device)
         if self._batch_ptr is not None:
             self._batch_ptr = torch.zeros(self._batch_ptr.shape[0], dtype=torch.int32, device=self.device)
@@ -324,6 +366,10 @@ class UniformGroup:
         return out
 
     def select(self, idx: list[int]) -> "UniformGroup":
+        span = _span(idx)
+        if span is not None:
+            return UniformGroup(dict(zip(self._tensors, _copies([v[span[0]: span[1]] for v in self._tensors.values()]))),
+                                len(idx), self.device)
         sel = torch.tensor(idx, dtype=torch.long, device=self.device)
         return UniformGroup({k: v.index_select(0, sel) for k, v in self._tensors.items()}, len(idx), self.device)
 
@@ -421,8 +467,10 @@ class UniformGroup:
         return self
 
     def zero(self) -> None:
-        for t in self._tensors.values():
-            t.zero_()
+        _zero_all(list(self._tensors.values()))
+        self._no_rows()
+
+    def _no_rows(self) -> None:
         self._n = 0
         self._counted = True
 
@@ -528,8 +576,10 @@ class Batch:
 
     def zero(self) -> None:
         """Back to zero systems; the storage is zeroed and kept (nvalchemi/data/batch.py:690-737)."""
-        for group in self._storage.groups.values():
-            group.zero()
+        groups = list(self._storage.groups.values())
+        _zero_all([t for group in groups for _, t in group.items()])
+        for group in groups:
+            group._no_rows() if isinstance(group, UniformGroup) else group._no_segments()
         self._drop_neighbor_stamps()
 
     def _drop_neighbor_stamps(self) -> None:
@@ -705,12 +755,13 @@ class Batch:
         groups: dict[str, Any] = {}
         atoms = self._atoms_group
         offset_diff = None
+        edges = self._edges_group
         if atoms is not None:
             new_atoms = atoms.select(ids)
-            sel = torch.tensor(ids, dtype=torch.long, device=self.device)
-            offset_diff = atoms.batch_ptr[sel] - new_atoms.batch_ptr[:-1]
+            if edges is not None and "neighbor_list" in edges:
+                sel = torch.tensor(ids, dtype=torch.long, device=self.device)
+                offset_diff = atoms.batch_ptr[sel] - new_atoms.batch_ptr[:-1]
             groups["atoms"] = new_atoms
-        edges = self._edges_group
         if edges is not None:
             new_edges = edges.select(ids)
             if "neighbor_list" in new_edges and offset_diff is not None:
@@ -755,12 +806,14 @@ class Batch:
         else:
             copy_mask = torch.zeros(n, device=device, dtype=torch.bool)
             object.__setattr__(src_batch, "_copied_mask", copy_mask)
-        levels = []
-        for mine, theirs in ((self._system_group, src_batch._system_group),
-                             (self._atoms_group, src_batch._atoms_group),
-                             (self._edges_group, src_batch._edges_group)):
-            if mine is not None and theirs is not None and len(mine.keys()) and len(theirs.keys()):
-                levels.append((mine, theirs))
+        atoms, edges = self._atoms_group, self._edges_group
+        n_before = len(atoms) if atoms is not None else 0
+        if self._put_together(src_batch, mask, copy_mask, dest_mask) is not None:
+            if copied_mask is not None and copy_mask is not copied_mask:
+                copied_mask.copy_(copy_mask)
+            self._put_finish(src_batch, copy_mask, n_before)
+            return
+        levels = self._shared_levels(src_batch)
         fit_mask = torch.ones(n, device=device, dtype=torch.bool)
         for mine, theirs in levels:
             level_fit = torch.empty(n, device=device, dtype=torch.bool)
@@ -770,13 +823,108 @@ class Batch:
         copy_mask.copy_(fit_mask)
         if copied_mask is not None and copy_mask is not copied_mask:
             copied_mask.copy_(copy_mask)
-        atoms, edges = self._atoms_group, self._edges_group
-        n_before = len(atoms) if atoms is not None else 0
         for mine, theirs in levels:
             if isinstance(mine, UniformGroup):
                 mine.put(theirs, copy_mask, copied_mask=copy_mask, dest_mask=dest_mask)
             else:
                 mine.put(theirs, copy_mask, copied_mask=copy_mask)
+        self._put_finish(src_batch, copy_mask, n_before)
+
+    def _shared_levels(self, src_batch: "Batch") -> list[tuple]:
+        """The levels that a put copies: both batches have tensors there."""
+        return [(mine, theirs) for mine, theirs in ((self._system_group, src_batch._system_group),
+                                                    (self._atoms_group, src_batch._atoms_group),
+                                                    (self._edges_group, src_batch._edges_group))
+                if mine is not None and theirs is not None and len(mine.keys()) and len(theirs.keys())]
+
+    def _put_together(self, src_batch: "Batch", mask: torch.Tensor, copy_mask: torch.Tensor, dest_mask: torch.Tensor | None, *,
+                      spare: int | None = None, max_masked: int = -1,
+                      longest: tuple[int, int] = (-1, -1)) -> tuple[int, ...] | None:
+        """:meth:`put` of every level and tensor in one plan and one copy, and one host read for all the counts.  ``None``,
+        with nothing done, where the general path has to take over: tensors elsewhere than on this device, not contiguous,
+        with gradients, of shapes or dtypes that do not match, a boundary tensor without headroom.
+
+        ``spare`` (systems the buffer holds): the boundary tensors are made anew with that headroom, whatever they had.
+        ``max_masked`` and ``longest`` (atoms, edges): more masked systems or a longer one refuse the call, nothing moves.
+        Returns (masked, most atoms, most edges, moved, accepted)."""
+        dev, n = self.device, src_batch.num_graphs
+        if (dev.type != "cuda" or n == 0 or src_batch is self or src_batch.device != mask.device
+                or torch.compiler.is_compiling()):
+            return None
+        plain = _lib.plain_on_device
+        if not (plain(mask, mask.device) and plain(copy_mask, mask.device) and mask.shape == copy_mask.shape == (n,)):
+            return None
+        dev = mask.device
+        fields, levels, segmented, n_slots, uniform = [], [], [], -1, None
+        if dest_mask is not None and not (plain(dest_mask, dev) and dest_mask.dtype == torch.bool and dest_mask.dim() == 1):
+            return None
+        for mine, theirs in self._shared_levels(src_batch):
+            if len(theirs) != n:
+                return None
+            rows = mine.capacity()
+            is_uniform = isinstance(mine, UniformGroup)
+            level = 0 if is_uniform else len(levels) + 1
+            count = len(fields)
+            for key in mine.keys():
+                if key not in theirs:
+                    continue
+                src_t, dest_t = theirs._tensors[key], mine._tensors[key]
+                if not is_uniform and (key in _NEIGHBOR_MATRIX_KEYS or src_t.dtype != dest_t.dtype
+                                       or src_t.dtype not in _BUFFER_DTYPES):
+                    continue
+                if is_uniform and src_t.shape[0] > n:
+                    src_t = src_t[:n]
+                if (not plain(src_t, dev) or not plain(dest_t, dev) or src_t.dtype != dest_t.dtype
+                        or src_t.shape[1:] != dest_t.shape[1:] or dest_t.shape[0] != rows
+                        or (is_uniform and src_t.shape[0] != n)):
+                    return None
+                row_bytes = math.prod(src_t.shape[1:]) * src_t.element_size()
+                if row_bytes == 0:
+                    return None
+                fields.append((src_t, dest_t, row_bytes, level, src_t.shape[0]))
+            if len(fields) == count:
+                return None
+            if is_uniform:
+                if dest_mask is not None and dest_mask.shape[0] != rows:
+                    return None
+                n_slots, uniform = rows, mine
+                continue
+            store, src_ptr, n_dest = mine._ptr_store(), theirs.batch_ptr, len(mine)
+            if not (plain(store, dev) and store.dtype == torch.int32 and plain(src_ptr, dev) and src_ptr.dtype == torch.int32):
+                return None
+            if (spare is None and store.shape[0] < n_dest + n + 2) or store.shape[0] < n_dest + 1:
+                return None
+            segmented.append((mine, n_dest))
+            levels.append((src_ptr, store, n_dest, rows, longest[0 if mine is self._atoms_group else 1]))
+        if (longest[0] >= 0 and self._atoms_group not in [m for m, _ in segmented]) or not segmented:
+            return None
+        ends = [8]
+        for _, _, n_dest, _, _ in levels:
+            ends.append(ends[-1] + n_dest + n)
+        out = torch.empty(ends[-1], dtype=torch.int32, device=dev)  # the counts, then the segments' lengths by level
+        news = [torch.empty(max(n_dest + n + 1, 0 if spare is None else spare + 2), dtype=torch.int32, device=dev)
+                for _, _, n_dest, _, _ in levels]
+        _lib.put_batch(fields, [(sp, store, news[q], out[ends[q]: ends[q + 1]], n_dest, rows, limit)
+                                for q, (sp, store, n_dest, rows, limit) in enumerate(levels)],
+                       mask, copy_mask, dest_mask if uniform is not None else None, n_slots, max_masked, out[:8])
+        host = out.tolist()
+        masked, moved, accepted = host[0], host[3], host[4]
+        if accepted:
+            for q, (mine, n_dest) in enumerate(segmented):
+                new_n = n_dest + moved
+                mine._batch_ptr = news[q][: new_n + 1] if spare is None else news[q][: max(spare, new_n) + 2]
+                mine.segment_lengths = out[ends[q]: ends[q] + new_n]
+                mine._over_allocated = True
+                mine._invalidate()
+                mine._lengths_host = host[ends[q]: ends[q] + new_n]
+            if uniform is not None and uniform._counted:
+                uniform._n += moved
+        most = {id(mine): host[1 + q] for q, (mine, _) in enumerate(segmented)}
+        return masked, most.get(id(self._atoms_group), 0), most.get(id(self._edges_group), 0), moved, accepted
+
+    def _put_finish(self, src_batch: "Batch", copy_mask: torch.Tensor, n_before: int) -> None:
+        device = self.device
+        atoms, edges = self._atoms_group, self._edges_group
         # the copied edges name atoms by their index in the source: move them to where the atoms went
         src_atoms, src_edges = src_batch._atoms_group, src_batch._edges_group
         if atoms is not None and src_atoms is not None and edges is not None and src_edges is not None \

@@ -128,22 +128,21 @@ class GPUBuffer(DataSink):
         if mask is None:
             mask = torch.ones(num_total, dtype=torch.bool, device=batch.device)
         self._ensure_buffer(template=batch)
+        if self._write_together(batch, mask):
+            return
         num_to_write = int(mask.sum().item())
         if num_to_write == 0:
             return
         current = len(self)
         if current + num_to_write > self._capacity:
-            raise RuntimeError(f"Buffer is full. Cannot add {num_to_write} samples to buffer "
-                               f"with {current}/{self._capacity} samples.")
+            self._refuse_systems(num_to_write, current)
         most_atoms = int(batch.num_nodes_per_graph[mask].max().item())
         if most_atoms > self._max_atoms:
-            raise RuntimeError(f"Atom capacity exceeded: a system has {most_atoms} atoms "
-                               f"but buffer max_atoms={self._max_atoms}")
+            self._refuse_atoms(most_atoms)
         if self._max_edges > 0 and batch.num_edges > 0:
             most_edges = int(batch.num_edges_per_graph[mask].max().item())
             if most_edges > self._max_edges:
-                raise RuntimeError(f"Edge capacity exceeded: a system has {most_edges} edges "
-                                   f"but buffer max_edges={self._max_edges}")
+                self._refuse_edges(most_edges)
         self._copied_mask = torch.zeros(num_total, dtype=torch.bool, device=self._device)
         self._restore_batch_ptr_capacity(incoming=num_total)
         self._buffer.put(batch, mask, copied_mask=self._copied_mask, dest_mask=self._dest_mask)
@@ -152,13 +151,53 @@ class GPUBuffer(DataSink):
         if placed != num_to_write:
             raise RuntimeError(f"GPUBuffer placed {placed} of {num_to_write} systems")
 
+    def _write_together(self, batch: Batch, mask: torch.Tensor) -> bool:
+        """The checks of :meth:`write`, the copy and the boundaries in two launches and one host read, where the batch's
+        tensors allow it (:meth:`Batch._put_together`)."""
+        count_edges = self._max_edges > 0 and batch._edges_group is not None and len(batch._edges_group)
+        if count_edges and (self._buffer._edges_group is None or not len(batch._edges_group.keys())):
+            return False
+        atoms = self._buffer._atoms_group
+        n_before, current = 0 if atoms is None else len(atoms), len(self)
+        copied = torch.zeros(mask.shape[0], dtype=torch.bool, device=self._device)
+        done = self._buffer._put_together(batch, mask, copied, self._dest_mask, spare=self._capacity,
+                                          max_masked=self._capacity - current,
+                                          longest=(self._max_atoms, self._max_edges if count_edges else -1))
+        if done is None:
+            return False
+        masked, most_atoms, most_edges, moved, accepted = done
+        if not accepted:
+            if current + masked > self._capacity:
+                self._refuse_systems(masked, current)
+            if most_atoms > self._max_atoms:
+                self._refuse_atoms(most_atoms)
+            self._refuse_edges(most_edges)
+        if masked:
+            self._copied_mask = copied
+            self._buffer._put_finish(batch, copied, n_before)
+            if moved != masked:
+                raise RuntimeError(f"GPUBuffer placed {moved} of {masked} systems")
+        return True
+
+    def _refuse_systems(self, num_to_write: int, current: int) -> None:
+        raise RuntimeError(f"Buffer is full. Cannot add {num_to_write} samples to buffer "
+                           f"with {current}/{self._capacity} samples.")
+
+    def _refuse_atoms(self, most_atoms: int) -> None:
+        raise RuntimeError(f"Atom capacity exceeded: a system has {most_atoms} atoms "
+                           f"but buffer max_atoms={self._max_atoms}")
+
+    def _refuse_edges(self, most_edges: int) -> None:
+        raise RuntimeError(f"Edge capacity exceeded: a system has {most_edges} edges "
+                           f"but buffer max_edges={self._max_edges}")
+
     def read(self) -> Batch:
         """The stored systems as a batch with tight tensors.  (When the buffer is full the
         reference returns a clone of the whole padded buffer, sinks.py:455-457; the systems are the
         same.)"""
         if self._buffer is None or len(self) == 0:
             raise RuntimeError("Cannot read from empty buffer.")
-        return self._buffer.index_select(torch.arange(len(self), dtype=torch.long, device=self._device))
+        return self._buffer.index_select(range(len(self)))
 
     def zero(self) -> None:
         if self._dest_mask is not None:
