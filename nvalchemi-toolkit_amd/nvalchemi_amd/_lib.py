@@ -788,7 +788,14 @@ def plain_on_device(t: torch.Tensor, device: torch.device) -> bool:
     """A tensor whose rows may be moved through its pointer: an ordinary contiguous one of a supported dtype on ``device``
     that no gradient is recorded for."""
     return (type(t) is torch.Tensor and t.is_cuda and t.device == device and t.dtype in BUFFER_DTYPES
-            and not t.requires_grad and t.is_contiguous())
+            and not t.requires_grad and t.is_contiguous() and not t.is_neg())
+
+
+def plainly_eager() -> bool:
+    """No tracing, functorch transform, forward-mode level or dispatch mode is active: what is done through a tensor's pointer
+    is all there is to do (a tangent, a batch dimension or a recorded operation would be lost)."""
+    return (not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
 
 
 def put_batch(fields, levels, mask, copied, dest_mask, n_slots: int, max_masked: int, counts) -> None:

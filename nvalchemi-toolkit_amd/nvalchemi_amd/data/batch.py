@@ -43,7 +43,7 @@ def _span(idx: list[int]) -> tuple[int, int] | None:
 def _copies(tensors: list[torch.Tensor]) -> list[torch.Tensor]:
     """Contiguous copies (one launch for tensors on the GPU that need no gradient)."""
     dev = tensors[0].device if tensors else None
-    if dev is None or dev.type != "cuda" or torch.compiler.is_compiling() \
+    if dev is None or dev.type != "cuda" or not _lib.plainly_eager() \
             or not all(_lib.plain_on_device(t, dev) for t in tensors):
         return [t.clone(memory_format=torch.contiguous_format) for t in tensors]
     out = [torch.empty(t.shape, dtype=t.dtype, device=dev) for t in tensors]
@@ -54,7 +54,7 @@ def _copies(tensors: list[torch.Tensor]) -> list[torch.Tensor]:
 def _zero_all(tensors: list[torch.Tensor]) -> None:
     """``zero_()`` of every tensor (one launch where :func:`_copies` makes one)."""
     dev = tensors[0].device if tensors else None
-    if dev is None or dev.type != "cuda" or torch.compiler.is_compiling() \
+    if dev is None or dev.type != "cuda" or not _lib.plainly_eager() \
             or not all(_lib.plain_on_device(t, dev) for t in tensors):
         for t in tensors:
             t.zero_()
@@ -849,7 +849,7 @@ class Batch:
         Returns (masked, most atoms, most edges, moved, accepted)."""
         dev, n = self.device, src_batch.num_graphs
         if (dev.type != "cuda" or n == 0 or src_batch is self or src_batch.device != mask.device
-                or torch.compiler.is_compiling()):
+                or not _lib.plainly_eager()):
             return None
         plain = _lib.plain_on_device
         if not (plain(mask, mask.device) and plain(copy_mask, mask.device) and mask.shape == copy_mask.shape == (n,)):
