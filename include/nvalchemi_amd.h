@@ -455,6 +455,18 @@ int32_t nvamd_nhc_position_update_f64(double* positions, const double* velocitie
 int32_t nvamd_nl_status(void* workspace, size_t workspace_bytes, int32_t n_atoms, int32_t n_systems,
                         int32_t* status, int32_t clear, void* stream);
 
+/* What compute_neighbors (nvalchemi/neighbors.py:253-277) reads on the host after a build, at one go: summary (4) i64 on the
+ * device = largest count, sum of the counts, status bits of the last build, of all builds since they were cleared. */
+int32_t nvamd_nl_summary(const void* workspace, size_t workspace_bytes, const int32_t* num_neighbors, int32_t n_atoms,
+                         int32_t n_systems, int64_t* summary, void* stream);
+
+/* Slots [num_neighbors[i], max_neighbors) of every row set to fill_value, their shifts (may be null) to zero. */
+int32_t nvamd_nl_pad_rows(const int32_t* num_neighbors, int32_t n_atoms, int32_t max_neighbors, int32_t fill_value,
+                          int32_t* neighbor_matrix, int32_t* neighbor_matrix_shifts, void* stream);
+
+/* stress = -virial / |det cell| (nvalchemi/models/lj.py adapt_output), (n_systems, 3, 3) each. */
+int32_t nvamd_stress(const float* virial, const float* cell, int32_t n_systems, float* stress, void* stream);
+
 /* Atom indices in the cell order of the neighbor build that last used this workspace with the same
  * n_atoms / n_systems: atom_order[k] for k in a system's range [batch_ptr[s], batch_ptr[s+1]) are that
  * system's atoms, cell by cell.  With rebuild_flags, only the ranges of flagged systems are written

@@ -49,6 +49,20 @@ struct Float3 {
     float x, y, z;
 };
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// Words [begin, end) of a row of int32 set to one value by a wave, in 16-byte stores between the aligned addresses.
+// (non-temporal: nobody reads the padding back, and it is most of what is written)
+__device__ __forceinline__ void fill_words(int32_t* row, int begin, int end, int value, int lane) {
+    const int to_line = (int)((0 - (reinterpret_cast<uintptr_t>(row + begin) >> 2)) & 3);
+    const int first = begin + to_line < end ? begin + to_line : end;
+    const int last = first + ((end - first) & ~3);
+    if (begin + lane < first) __builtin_nontemporal_store(value, row + begin + lane);
+    const v4i v = {value, value, value, value};
+    for (int k = first + 4 * lane; k < last; k += 4 * 64) __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(row + k));
+    if (last + lane < end) __builtin_nontemporal_store(value, row + last + lane);
+}
+
 // wave-wide sum of a double via xor shuffles (all 64 lanes end with the total)
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

@@ -64,6 +64,20 @@ __global__ __launch_bounds__(kBlock) void coo_fill_kernel(const int32_t* __restr
     }
 }
 
+// The rows of a matrix behind their entries, a wave per row, in 16-byte stores.  (Padding the rows once the build has shown
+// that they are wide enough, instead of filling both tensors before it, and reading what the build found at one go: 64 boxes of
+// 1000 atoms with rows of 784 slots, 800 MB of padding, bound by these stores, 398 -> 350 us for list and evaluation; 512 cells
+// of 8-500 atoms 418 -> 253 us; edge lists, which need no padding, of 1024 cells 383 -> 312 us.)
+__global__ __launch_bounds__(kBlock) void pad_rows_kernel(const int32_t* __restrict__ nn, int n_atoms, int K, int fill,
+                                                          int32_t* __restrict__ nm, int32_t* __restrict__ shifts) {
+    const int i = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)kBlock + threadIdx.x) / 64));
+    if (i >= n_atoms) return;
+    const int n = nn[i], lane = lane_id();
+    const int kept = n < 0 ? 0 : (n < K ? n : K);
+    fill_words(nm + (size_t)i * K, kept, K, fill, lane);
+    if (shifts) fill_words(shifts + (size_t)i * K * 3, 3 * kept, 3 * K, 0, lane);
+}
+
 // the same two numbers where there is nothing to fill
 __global__ void coo_count_kernel(const int32_t* __restrict__ edge_ptr, int n_atoms, long long cap,
                                  int32_t* __restrict__ counts) {
@@ -143,4 +157,18 @@ NVAMD_EXPORT int32_t nvamd_nl_coo_from_matrix(const int32_t* neighbor_matrix, co
     if (rc != NVAMD_OK) return rc;
     return fill(neighbor_matrix, neighbor_matrix_shifts, edge_ptr, n_atoms, max_neighbors, edge_capacity, neighbor_list,
                 neighbor_list_shifts, counts, static_cast<hipStream_t>(stream));
+}
+
+NVAMD_EXPORT int32_t nvamd_nl_pad_rows(const int32_t* num_neighbors, int32_t n_atoms, int32_t max_neighbors, int32_t fill_value,
+                                       int32_t* neighbor_matrix, int32_t* neighbor_matrix_shifts, void* stream) {
+    if (n_atoms < 0 || max_neighbors < 0 || (long long)max_neighbors * 3 > 0x7fffffffLL)
+        return fail(NVAMD_ERR_INVALID_ARGUMENT, "pad rows: bad size");
+    if (n_atoms == 0 || max_neighbors == 0) return NVAMD_OK;
+    if (!num_neighbors || !neighbor_matrix) return fail(NVAMD_ERR_INVALID_ARGUMENT, "pad rows: null buffer");
+    const size_t threads = (size_t)n_atoms * 64;
+    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((threads + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                       static_cast<hipStream_t>(stream), num_neighbors, n_atoms, max_neighbors, fill_value, neighbor_matrix,
+                       neighbor_matrix_shifts);
+    NVAMD_LAUNCH_CHECK("pad rows launch");
+    return NVAMD_OK;
 }

@@ -22,20 +22,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kInFlight = 4;  // steps of 64 slots whose loads are in flight together
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-
-// Words [begin, end) of a row of int32 set to one value by a wave, in 16-byte stores between the aligned addresses.
-// (non-temporal: nobody reads the padding back, and it is most of what is written)
-__device__ __forceinline__ void fill_words(int32_t* row, int begin, int end, int value, int lane) {
-    const int to_line = (int)((0 - (reinterpret_cast<uintptr_t>(row + begin) >> 2)) & 3);
-    const int first = begin + to_line < end ? begin + to_line : end;
-    const int last = first + ((end - first) & ~3);
-    if (begin + lane < first) __builtin_nontemporal_store(value, row + begin + lane);
-    const v4i v = {value, value, value, value};
-    for (int k = first + 4 * lane; k < last; k += 4 * kWave) __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(row + k));
-    if (last + lane < end) __builtin_nontemporal_store(value, row + last + lane);
-}
-
 // The shift of a padding slot is not read (it is zero in the result whatever it was), the four steps' loads go out
 // together, and the padding leaves in 16-byte stores: 64 000 rows of 272 slots (78 valid) take 87 us instead of 124, 60 when
 // they have just been read (408 MB have to move: 4.7 TB/s).

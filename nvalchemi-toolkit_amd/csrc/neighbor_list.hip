@@ -1642,6 +1642,46 @@ __global__ void nl_status_kernel(NlHeader* hdr, int32_t* out, int clear) {
     }
 }
 
+// what a caller that sizes its rows by the result has to know: the largest count, the number of entries, the status bits
+__global__ void nl_summary_begin_kernel(const NlHeader* hdr, long long* out) {
+    out[0] = 0;
+    out[1] = 0;
+    out[2] = hdr->error[hdr->flip ^ 1];
+    out[3] = hdr->sticky | hdr->error[0] | hdr->error[1];
+}
+
+__global__ __launch_bounds__(kBlock) void nl_summary_kernel(const int32_t* __restrict__ nn, int n_atoms, long long* out) {
+    __shared__ int sh_most;
+    __shared__ unsigned long long sh_sum;
+    if (threadIdx.x == 0) {
+        sh_most = 0;
+        sh_sum = 0;
+    }
+    __syncthreads();
+    int most = 0;
+    long long sum = 0;
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n_atoms; i += (long long)gridDim.x * kBlock) {
+        const int c = nn[i];
+        most = most > c ? most : c;
+        sum += c;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const int m = __shfl_xor(most, o, kWave);
+        most = most > m ? most : m;
+        sum += __shfl_xor(sum, o, kWave);
+    }
+    if (lane_id() == 0) {
+        atomicMax(&sh_most, most);
+        atomicAdd(&sh_sum, (unsigned long long)sum);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(out, (long long)sh_most);
+        atomicAdd(reinterpret_cast<unsigned long long*>(out + 1), sh_sum);
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void nl_atom_order_kernel(const float4* __restrict__ sorted_pos,
                                                                const int32_t* __restrict__ bidx,
                                                                const uint8_t* __restrict__ flags, int n_atoms,
@@ -1686,6 +1726,27 @@ NVAMD_EXPORT int32_t nvamd_nl_status(void* workspace, size_t workspace_bytes, in
     hipLaunchKernelGGL(nl_status_kernel, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), ws.hdr, status,
                        clear ? 1 : 0);
     NVAMD_LAUNCH_CHECK("nl status launch");
+    return NVAMD_OK;
+}
+
+NVAMD_EXPORT int32_t nvamd_nl_summary(const void* workspace, size_t workspace_bytes, const int32_t* num_neighbors,
+                                      int32_t n_atoms, int32_t n_systems, int64_t* summary, void* stream) {
+    if (n_atoms < 0 || n_systems < 0 || !summary || (n_atoms > 0 && !num_neighbors))
+        return fail(NVAMD_ERR_INVALID_ARGUMENT, "nl summary: bad argument");
+    size_t need = carve(nullptr, nullptr, n_atoms, n_systems);
+    if (!workspace || workspace_bytes < need)
+        return fail(NVAMD_ERR_WORKSPACE_TOO_SMALL, "nl summary: workspace %zu < %zu bytes", workspace_bytes, need);
+    NlWorkspace ws;
+    carve(&ws, static_cast<char*>(const_cast<void*>(workspace)), n_atoms, n_systems);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    long long* out = reinterpret_cast<long long*>(summary);
+    hipLaunchKernelGGL(nl_summary_begin_kernel, dim3(1), dim3(1), 0, st, ws.hdr, out);
+    if (n_atoms > 0) {
+        // four counts per lane, up to two workgroups per CU
+        const int blocks = (n_atoms + 4 * kBlock - 1) / (4 * kBlock);
+        hipLaunchKernelGGL(nl_summary_kernel, dim3(blocks < 512 ? blocks : 512), dim3(kBlock), 0, st, num_neighbors, n_atoms, out);
+    }
+    NVAMD_LAUNCH_CHECK("nl summary launch");
     return NVAMD_OK;
 }
 

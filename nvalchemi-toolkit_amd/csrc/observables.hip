@@ -125,6 +125,17 @@ int32_t run(const float* values, const float* masses, const int32_t* bidx, int32
     return NVAMD_OK;
 }
 
+// stress = -virial / |det cell|, a lane per component (the determinant in float64: it is nine products)
+__global__ __launch_bounds__(kBlock) void stress_kernel(const float* __restrict__ virial, const float* __restrict__ cell, int n,
+                                                        float* __restrict__ stress) {
+    const int t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= 9 * n) return;
+    const float* c = cell + (size_t)(t / 9) * 9;
+    const double a = c[0], b = c[1], d = c[2], e = c[3], f = c[4], g = c[5], h = c[6], k = c[7], l = c[8];
+    const float volume = (float)fabs(a * (f * l - g * k) - b * (e * l - g * h) + d * (e * k - f * h));
+    stress[t] = -virial[t] / volume;
+}
+
 }  // namespace
 }  // namespace nvamd
 
@@ -150,4 +161,14 @@ NVAMD_EXPORT int32_t nvamd_kinetic_energy(const float* velocities, const float* 
     if (n_atoms > 0 && !masses) return fail(NVAMD_ERR_INVALID_ARGUMENT, "kinetic energy: null masses");
     return run(velocities, masses, batch_idx, n_atoms, n_systems, kOpKinetic, kinetic_energy, workspace,
                workspace_bytes, stream, "kinetic energy");
+}
+
+NVAMD_EXPORT int32_t nvamd_stress(const float* virial, const float* cell, int32_t n_systems, float* stress, void* stream) {
+    if (n_systems < 0 || n_systems > 0x7fffffff / 9) return fail(NVAMD_ERR_INVALID_ARGUMENT, "stress: bad number of systems");
+    if (n_systems == 0) return NVAMD_OK;
+    if (!virial || !cell || !stress) return fail(NVAMD_ERR_INVALID_ARGUMENT, "stress: null buffer");
+    hipLaunchKernelGGL(stress_kernel, dim3((unsigned)((9LL * n_systems + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                       static_cast<hipStream_t>(stream), virial, cell, n_systems, stress);
+    NVAMD_LAUNCH_CHECK("stress launch");
+    return NVAMD_OK;
 }

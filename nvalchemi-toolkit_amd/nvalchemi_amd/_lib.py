@@ -99,6 +99,9 @@ _SIGNATURES = {
     "nvamd_defrag_per_system": (_i32, [_vp, _vp, _i32, _c.c_int64, _vp, _c.c_size_t, _vp]),
     "nvamd_put_masked_segmented": (_i32, [_vp] * 5 + [_i32, _i32, _vp, _vp, _i32, _i32, _c.c_int64, _vp,
                                           _c.c_size_t, _vp]),
+    "nvamd_nl_summary": (_i32, [_vp, _c.c_size_t, _vp, _i32, _i32, _vp, _vp]),
+    "nvamd_nl_pad_rows": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp]),
+    "nvamd_stress": (_i32, [_vp, _vp, _i32, _vp, _vp]),
     "nvamd_put_batch": (_i32, [_c.POINTER(PutField), _i32, _c.POINTER(PutLevel), _i32, _vp, _vp, _vp, _i32, _i32, _i32, _vp,
                                _vp, _c.c_size_t, _vp]),
     "nvamd_copy_ranges": (_i32, [_c.POINTER(_vp), _c.POINTER(_vp), _c.POINTER(_c.c_int64), _i32, _vp]),
@@ -338,6 +341,27 @@ def nl_status(n_atoms: int, n_systems: int, device, clear: bool = False,
     _check(lib.nvamd_nl_status(ws.data_ptr(), ws.numel() * ws.element_size(), int(n_atoms), int(n_systems),
                                out.data_ptr(), int(bool(clear)), _stream(torch.device(device))), "nvamd_nl_status")
     return out
+
+
+def nl_summary(num_neighbors, n_systems: int) -> tuple[int, int, int, int]:
+    """(largest count, sum of the counts, status bits of the last build, of all since they were cleared) after a build
+    through the workspace of this device and stream, in one host read."""
+    N, device = num_neighbors.shape[0], num_neighbors.device
+    ws = workspaces.get(device, "nl", nl_workspace_bytes(N, n_systems))
+    out = torch.empty(4, dtype=torch.int64, device=device)
+    _check(library().nvamd_nl_summary(ws.data_ptr(), ws.numel(), _dev(num_neighbors, "num_neighbors", torch.int32, (N,)), N,
+                                      n_systems, out.data_ptr(), _stream(device)), "nvamd_nl_summary")
+    return tuple(out.tolist())
+
+
+def nl_pad_rows(num_neighbors, fill_value: int, neighbor_matrix, neighbor_matrix_shifts=None) -> None:
+    """Padding behind the entries of every row: ``fill_value``, and zero shifts."""
+    N, K = neighbor_matrix.shape
+    _check(library().nvamd_nl_pad_rows(
+        _dev(num_neighbors, "num_neighbors", torch.int32, (N,)), N, K, fill_value,
+        _dev(neighbor_matrix, "neighbor_matrix", torch.int32, (N, K)),
+        _opt(neighbor_matrix_shifts, "neighbor_matrix_shifts", torch.int32, (N, K, 3)),
+        _stream(neighbor_matrix.device)), "nvamd_nl_pad_rows")
 
 
 def nl_edge_ptr(num_neighbors, max_neighbors, edge_ptr) -> None:
@@ -782,6 +806,15 @@ def defrag_segmented(source, source_batch_ptr, source_data_copied, num_kept) -> 
         sp, _dev(source_batch_ptr, "source_batch_ptr", torch.int32, (n + 1,)),
         _mask(source_data_copied, "source_data_copied", n), _dev(num_kept, "num_kept", torch.int32, (1,)),
         n, rows, rb, ws.data_ptr(), ws.numel(), _stream(source.device)), "nvamd_defrag_segmented")
+
+
+def stress_from_virial(virial, cell) -> torch.Tensor:
+    """``-virial / |det cell|`` of float32 ``(B, 3, 3)`` tensors."""
+    B = virial.shape[0]
+    out = torch.empty(B, 3, 3, dtype=torch.float32, device=virial.device)
+    _check(library().nvamd_stress(_dev(virial, "virial", torch.float32, (B, 3, 3)), _dev(cell, "cell", torch.float32, (B, 3, 3)),
+                                  B, out.data_ptr(), _stream(virial.device)), "nvamd_stress")
+    return out
 
 
 def plain_on_device(t: torch.Tensor, device: torch.device) -> bool:

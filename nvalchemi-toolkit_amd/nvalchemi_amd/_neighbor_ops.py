@@ -121,7 +121,7 @@ _last_edge_count: dict[tuple, int] = {}
 
 def get_neighbor_list_from_neighbor_matrix(neighbor_matrix: torch.Tensor, num_neighbors: torch.Tensor,
                                            neighbor_shift_matrix: torch.Tensor | None = None,
-                                           fill_value: int | None = None):
+                                           fill_value: int | None = None, n_edges: int | None = None):
     """Dense -> COO in row-major order.  Returns ``(edges (2,E) int32, edge_ptr (N+1) int32[,
     shifts (E,3) int32])`` like the reference's helper (the caller transposes ``[0]``).
 
@@ -129,7 +129,8 @@ def get_neighbor_list_from_neighbor_matrix(neighbor_matrix: torch.Tensor, num_ne
     sized by the edge count of the previous conversion of a matrix of this shape (plus headroom);
     the host then reads the count once, to cut the views to size (tensor shapes live on the host:
     the reference's helper waits for the same number), and repeats the call with larger buffers
-    only if they were too small."""
+    only if they were too small.  With ``n_edges`` (the sum of the counts, none of them above K) the buffers are made for
+    them and nothing is read."""
     N, K = neighbor_matrix.shape
     dev = neighbor_matrix.device
     key = (dev.index, N, K)
@@ -137,6 +138,10 @@ def get_neighbor_list_from_neighbor_matrix(neighbor_matrix: torch.Tensor, num_ne
     cap = N * K if guess is None else min(N * K, int(guess * 1.05) + 1024)
     if guess is None and N * K > (1 << 22):
         cap = 0  # a first conversion of a large matrix: count first, rather than allocate N x K edges
+    if n_edges is not None:
+        # (rounded up by an eighth at most: inputs of about the same size then find each other's memory in the allocator)
+        step = 1 << max(n_edges.bit_length() - 4, 0)
+        cap = -(-n_edges // step) * step
     edge_ptr = torch.empty(N + 1, dtype=torch.int32, device=dev)
     counts = torch.empty(2, dtype=torch.int32, device=dev)
     want_shifts = neighbor_shift_matrix is not None
@@ -144,11 +149,15 @@ def get_neighbor_list_from_neighbor_matrix(neighbor_matrix: torch.Tensor, num_ne
         edges = torch.empty((cap, 2), dtype=torch.int32, device=dev)
         shifts = torch.empty((cap, 3), dtype=torch.int32, device=dev) if want_shifts else None
         _lib.nl_coo_from_matrix(neighbor_matrix, neighbor_shift_matrix, num_neighbors, edge_ptr, edges, shifts, counts)
+        if n_edges is not None:
+            E = n_edges
+            break
         E, over = (int(v) for v in counts.tolist())
         if not over:
             break
         cap = E
-    _last_edge_count[key] = E
+    if n_edges is None:
+        _last_edge_count[key] = E
     edges = edges[:E]
     if not want_shifts:
         return edges.T, edge_ptr

@@ -16,6 +16,7 @@ from typing import Any
 import torch
 from torch import nn
 
+from .. import _lib
 from ..data import AtomicData, Batch
 from ._ops.lj import lj_energy_forces_system_batch
 from .base import BaseModelMixin, ModelConfig, NeighborConfig, NeighborListFormat
@@ -115,8 +116,13 @@ class LennardJonesModelWrapper(nn.Module, BaseModelMixin):
             if "virial" in model_output:
                 if not hasattr(data, "cell") or data.cell is None:
                     raise ValueError("stress output requires cell for volume computation")
-                volume = torch.det(data.cell).abs().view(-1, 1, 1)
-                output["stress"] = -model_output["virial"] / volume
+                virial, cell = model_output["virial"], data.cell
+                if (_lib.plainly_eager() and cell.dtype == torch.float32 and virial.dtype == torch.float32
+                        and cell.shape == virial.shape and _lib.plain_on_device(cell, virial.device)
+                        and _lib.plain_on_device(virial, virial.device)):
+                    output["stress"] = _lib.stress_from_virial(virial, cell)
+                else:
+                    output["stress"] = -virial / torch.det(cell).abs().view(-1, 1, 1)
             elif "stress" in model_output:
                 output["stress"] = model_output["stress"]
             else:

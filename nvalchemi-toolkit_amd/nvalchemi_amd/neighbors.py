@@ -11,7 +11,8 @@ from __future__ import annotations
 
 import torch
 
-from ._neighbor_ops import estimate_max_neighbors, get_neighbor_list_from_neighbor_matrix, neighbor_list
+from . import _lib
+from ._neighbor_ops import ceil16, estimate_max_neighbors, get_neighbor_list_from_neighbor_matrix, neighbor_list
 from .data.batch import Batch, SegmentedGroup
 from .models.base import NeighborConfig, NeighborListFormat
 
@@ -24,10 +25,11 @@ def _raise_on_truncated_search(n_atoms: int, n_systems: int, device, cutoff: flo
     Called where the host waits for the device anyway."""
     if n_atoms == 0:
         return
-    from . import _lib
+    _raise_on_status(int(_lib.nl_status(n_atoms, n_systems, device)[0]), cutoff)
 
-    now = int(_lib.nl_status(n_atoms, n_systems, device)[0])
-    if now & _lib.NL_STATUS_CELL_TOO_THIN:
+
+def _raise_on_status(status: int, cutoff: float) -> None:
+    if status & _lib.NL_STATUS_CELL_TOO_THIN:
         raise ValueError(f"a periodic cell is singular or thinner than cutoff / 32 (cutoff {cutoff}): "
                          "its neighbor list would be truncated")
 
@@ -35,16 +37,17 @@ def _raise_on_truncated_search(n_atoms: int, n_systems: int, device, cutoff: flo
 def _write_neighbor_data_to_batch(batch: Batch, neighbor_matrix: torch.Tensor, num_neighbors: torch.Tensor,
                                   neighbor_matrix_shifts: torch.Tensor | None,
                                   format: NeighborListFormat, cutoff: float,
-                                  search_cutoff: float | None = None) -> None:
+                                  search_cutoff: float | None = None, n_edges: int | None = None) -> None:
     """Publish neighbor data on *batch* (MATRIX: three atom keys; COO: a new edges group
     with per-graph edge counts) and stamp the cutoff.  ``search_cutoff`` is the radius the
     matrix was actually searched with (cutoff plus skin, a full list); it is kept on the batch
     together with the identity of the matrix so that a pair kernel may derive shifts from
-    positions where the cell is wide enough."""
+    positions where the cell is wide enough.  ``n_edges``: the sum of the counts, where the caller knows it and that no
+    row overflowed."""
     object.__setattr__(batch, "_neighbor_search_cutoff", None)
     if format == NeighborListFormat.COO:
         coo = get_neighbor_list_from_neighbor_matrix(neighbor_matrix, num_neighbors,
-                                                     neighbor_matrix_shifts, fill_value=batch.num_nodes)
+                                                     neighbor_matrix_shifts, fill_value=batch.num_nodes, n_edges=n_edges)
         edges = coo[0].T  # (E, 2) int32, already laid out row by row
         if not edges.is_contiguous():
             edges = edges.contiguous()
@@ -73,6 +76,11 @@ def _write_neighbor_data_to_batch(batch: Batch, neighbor_matrix: torch.Tensor, n
     batch._neighbor_list_cutoff = cutoff
 
 
+def _any(flags: torch.Tensor) -> bool:
+    """``bool(flags.any())``; a short tensor is read whole, which takes a launch less than reducing it first."""
+    return bool((flags.cpu() if flags.numel() <= 1 << 16 else flags).any())
+
+
 def compute_neighbors(batch: Batch, cutoff: float | None = None, *, config: NeighborConfig | None = None,
                       format: NeighborListFormat = NeighborListFormat.MATRIX,
                       max_neighbors: int | None = None, half_list: bool = False) -> None:
@@ -96,7 +104,7 @@ def compute_neighbors(batch: Batch, cutoff: float | None = None, *, config: Neig
     device = batch.device
     pbc = getattr(batch, "pbc", None)
     cell = getattr(batch, "cell", None)
-    if pbc is not None and not bool(pbc.any()):
+    if pbc is not None and not _any(pbc):
         pbc = None
         cell = None
     if cell is None:
@@ -111,21 +119,30 @@ def compute_neighbors(batch: Batch, cutoff: float | None = None, *, config: Neig
     batch_ptr = batch.batch_ptr.to(torch.int32)
     batch_idx = batch.batch_idx.to(torch.int32)
 
+    # Rows are allocated as they are: the build writes a row's entries (the counts say that no row holds any yet), and the
+    # padding of a matrix is written when the rows are known to be wide enough.  An edge list needs none.
+    most, n_edges, sized = 0, 0, N == 0
     while True:
-        nb_matrix = torch.full((N, max_neighbors), N, dtype=torch.int32, device=device)
+        nb_matrix = torch.empty((N, max_neighbors), dtype=torch.int32, device=device)
         nb_counts = torch.zeros(N, dtype=torch.int32, device=device)
         nb_shifts = None
         if pbc is not None:
-            nb_shifts = torch.zeros(N, max_neighbors, 3, dtype=torch.int32, device=device)
+            nb_shifts = torch.empty((N, max_neighbors, 3), dtype=torch.int32, device=device)
         neighbor_list(positions=batch.positions, cutoff=cutoff, cell=cell, pbc=pbc,
                       max_neighbors=max_neighbors, half_fill=half_list, batch_ptr=batch_ptr,
                       batch_idx=batch_idx, neighbor_matrix=nb_matrix, num_neighbors=nb_counts,
                       neighbor_matrix_shifts=nb_shifts, rebuild_flags=None, tail_mode=0)
-        actual_max = int(nb_counts.max()) if N > 0 else 0
-        if actual_max < max_neighbors:
+        if not sized:
+            most, n_edges, status, _ = _lib.nl_summary(nb_counts, batch.num_graphs)
+            _raise_on_status(status, cutoff)
+            sized = True
+        if most < max_neighbors:
             break
-        max_neighbors = int(actual_max * 1.5) + 1
-    _raise_on_truncated_search(N, batch.num_graphs, device, cutoff)
+        # (a matrix gets the headroom that its callers know; the rows behind an edge list are scratch, and rows without
+        # room to spare are a third less memory to touch)
+        max_neighbors = ceil16(most + 1) if format == NeighborListFormat.COO else int(most * 1.5) + 1
+    if format != NeighborListFormat.COO and N > 0:
+        _lib.nl_pad_rows(nb_counts, N, nb_matrix, nb_shifts)
 
     _write_neighbor_data_to_batch(batch, nb_matrix, nb_counts, nb_shifts, format, cutoff,
-                                  search_cutoff=None if half_list else cutoff)
+                                  search_cutoff=None if half_list else cutoff, n_edges=n_edges)
