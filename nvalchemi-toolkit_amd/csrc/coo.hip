@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kBlock) void coo_fill_kernel(const int32_t* __restr
 // The rows of a matrix behind their entries, a wave per row, in 16-byte stores.  (Padding the rows once the build has shown
 // that they are wide enough, instead of filling both tensors before it, and reading what the build found at one go: 64 boxes of
 // 1000 atoms with rows of 784 slots, 800 MB of padding, bound by these stores, 398 -> 350 us for list and evaluation; 512 cells
-// of 8-500 atoms 418 -> 253 us; edge lists, which need no padding, of 1024 cells 383 -> 312 us.)
+// of 8-500 atoms 418 -> 253 us; edge lists, which need no padding, of 1024 cells 383 -> 300 us.)
 __global__ __launch_bounds__(kBlock) void pad_rows_kernel(const int32_t* __restrict__ nn, int n_atoms, int K, int fill,
                                                           int32_t* __restrict__ nm, int32_t* __restrict__ shifts) {
     const int i = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)kBlock + threadIdx.x) / 64));
